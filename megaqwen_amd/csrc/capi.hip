@@ -637,7 +637,7 @@ int mq_flash_attn_bhwd(const void* d_q, const void* d_k, const void* d_v, void* 
                 workspace_bytes);
   const float scale_log2 = (float)((double)scale * 1.4426950408889634);
   const int rc = mq_launch_flash_attn_bhwd(d_q, d_k, d_v, d_out, batch * heads, seq_len,
-                                           dtype == MQ_DTYPE_F16, scale_log2, d_workspace,
+                                           dtype == MQ_DTYPE_F16, scale_log2,
                                            static_cast<hipStream_t>(stream));
   return rc == 0 ? MQ_OK : fail(MQ_ERR_HIP, "launch failed (%s)", hipGetErrorString(hipGetLastError()));
 }

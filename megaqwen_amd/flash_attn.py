@@ -68,8 +68,8 @@ def flash_attn_bhwd(
     ws_bytes = lib.mq_flash_attn_workspace_bytes(b, h, t, d)
     if ws_bytes == 0:
         _lib.check(_lib.MQ_ERR_INVALID_ARG)
-    # K and V^T in MFMA-operand order, written and consumed within the call (stream-ordered, so
-    # the caching allocator may hand the block out again once the call is queued)
+    # the scratch the C interface asks for (stream-ordered, so the caching allocator may hand the
+    # block out again once the call is queued)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
     with torch.cuda.device(q.device):
         stream = torch.cuda.current_stream(q.device).cuda_stream

@@ -75,6 +75,49 @@ def test_peaked_softmax(dtype):
     _check(out.cpu(), q, k, v)
 
 
+# (batch * heads, T): both query-block widths (32 queries per wave for the small grids, 64 once
+# 32-query workgroups exceed one round of the chip) at the edges of a key tile, of a query block
+# and of the four waves' ranges (waves without a tile, one tile each, uneven ranges)
+@pytest.mark.parametrize("bh,t", [(3, 31), (3, 32), (3, 33), (2, 64), (2, 65), (3, 127), (2, 129),
+                                  (1, 161), (400, 33), (400, 64), (220, 97), (160, 129),
+                                  (130, 191)])
+@pytest.mark.parametrize("dtype,scale", [(torch.bfloat16, 0.125), (torch.float16, -0.2),
+                                         (torch.bfloat16, 0.0)])
+def test_tile_edges(bh, t, dtype, scale):
+    q, k, v = _inputs((1, bh, t, 64), dtype, seed=bh + t)
+    out = _fa()(q.cuda(), k.cuda(), v.cuda(), scale=scale)
+    torch.cuda.synchronize()
+    _check(out.cpu(), q, k, v, scale)
+
+
+def test_unaligned_and_non_finite_inputs():
+    """Contiguous tensors that start 2 bytes into an allocation; an infinite value reaches only
+    its own dim's outputs, a NaN query only its own row, and the rows past T of the last key tile
+    (T % 32 != 0) add nothing."""
+    t = 70
+    q, k, v = _inputs((1, 2, t, 64), torch.bfloat16, seed=21)
+    dev = []
+    for x in (q, k, v):
+        buf = torch.zeros(x.numel() + 1, dtype=x.dtype, device="cuda")
+        buf[1:] = x.flatten().cuda()
+        dev.append(buf[1:].view(x.shape))
+    assert all(x.data_ptr() % 4 == 2 for x in dev)
+    out = _fa()(*dev)
+    torch.cuda.synchronize()
+    _check(out.cpu(), q, k, v)
+    want = out.cpu()
+    v2, q2 = v.clone(), q.clone()
+    v2[0, 0, t - 1, 5] = float("inf")
+    q2[0, 1, 3, 7] = float("nan")
+    got = _fa()(q2.cuda(), k.cuda(), v2.cuda()).cpu()
+    # (NaN instead of inf where the weight is a power of two: its lo part is 0, and 0 * inf is NaN)
+    assert not torch.isfinite(got[0, 0, :, 5]).any() and torch.isnan(got[0, 1, 3]).all()
+    assert torch.isinf(got[0, 0, :, 5]).float().mean() > 0.5
+    got[0, 0, :, 5] = want[0, 0, :, 5]
+    got[0, 1, 3] = want[0, 1, 3]
+    assert torch.equal(got, want)
+
+
 def test_deterministic_and_stream_ordered():
     q, k, v = (x.cuda() for x in _inputs((1, 14, 333, 64), torch.bfloat16, seed=3))
     s = torch.cuda.Stream()
