@@ -897,7 +897,9 @@ static void gemm(GemmArgs g, const MqPrefillBuffers& b, hipStream_t s) {
 static void pf_split_sizes(int max_n, size_t& part_bytes, size_t& tiles) {
   part_bytes = 0;
   tiles = 0;
-  for (int m = 1; m <= max_n; m = (m < 32 ? 32 : m + 32)) {
+  // plans change with the number of 32-row tiles: every multiple of 32 and, behind the last one,
+  // max_n itself
+  for (int m = 32;; m += 32) {
     const int mm = m > max_n ? max_n : m;
     const GemmPlan ps[] = {gemm_plan<EPI_QKV>(mm, MQ_QKV, MQ_H),
                            gemm_plan<EPI_RESID>(mm, MQ_H, MQ_QDIM),

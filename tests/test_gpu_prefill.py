@@ -256,3 +256,24 @@ def test_prefill_out_of_vocab_id_sets_device_error(small):
         dec.check()
     dec.reset()
     dec.check()
+
+
+@pytest.mark.parametrize("n", [33, 65, 90, 107, 131, 164, 224])
+def test_prefill_of_exactly_max_prefill_len(small, n):
+    """A decoder whose max_prefill_len is the prompt length itself (also off the 32-row tile
+    grid, where the split-K workspace must be sized for the last, partial tile) gives the logits
+    and cache rows of one with room to spare, bit for bit."""
+    dec, _, sp, w = small
+    from megaqwen_amd.decoder import MegakernelPrefillDecoder
+    toks = make_tokens(n, sp["vocab_size"], seed=n)
+    dec.reset()
+    _, want = dec.prefill_step_with_logits(toks)
+    tight = MegakernelPrefillDecoder(dec.embed_weight, dec.layer_weights, dec.final_norm_weight,
+                                     dec.lm_head_weight, dec.cos_table, dec.sin_table, 2, 640,
+                                     max_prefill_len=n)
+    for _ in range(2):
+        _, got = tight.prefill_step_with_logits(toks)
+        assert torch.equal(got, want)
+        assert torch.equal(tight.k_cache[:, :, :n], dec.k_cache[:, :, :n])
+        assert torch.equal(tight.v_cache[:, :, :n], dec.v_cache[:, :, :n])
+    dec.reset()
