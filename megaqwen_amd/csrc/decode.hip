@@ -156,7 +156,6 @@ struct RowSet {
 };
 
 typedef RowSet<MQ_H, 1, 3> QkvSet;      // 16 rows / workgroup at 256 workgroups
-typedef RowSet<MQ_QDIM, 2, 2> OSet;     //  4 rows x 2 segments
 typedef RowSet<MQ_H, 1, 4> GateUpSet;   // 12 gate + 12 up rows
 typedef RowSet<MQ_I, 2, 2> DownSet;     //  4 rows x 2 segments
 
@@ -899,31 +898,6 @@ MQ_DEV AttnItem attn_item(int wg, int nch, int cache_len) {
   it.p0 = it.c * clen;
   it.p1 = min(cache_len, it.p0 + clen);
   return it;
-}
-
-// ---------------------------------------------------------------------------- P3: O proj
-MQ_DEV void o_load(OSet& ws, const MqLayerW& w, int wg, int G) {
-  int r0, nr;
-  row_range(MQ_H, wg, G, r0, nr);
-  ws.load([&](int i) { return w.wo + (size_t)(r0 + i) * MQ_QDIM; }, nr);
-}
-// Input: att in LDS_IN; segment dot products -> LDS_PR.
-MQ_DEV void o_run(const OSet& ws, const MqLayerW& w, int wg, int G, float* lds) {
-  int r0, nr;
-  row_range(MQ_H, wg, G, r0, nr);
-  ws.compute([&](int i) { return w.wo + (size_t)(r0 + i) * MQ_QDIM; }, nr, lds + LDS_IN,
-             [&](int it, float v) { lds[LDS_PR + it] = v; });
-}
-// Sync-wave epilogue: lane t < nr (<= 64) holds the residual of hidden row r0 + t in `res`
-// and leaves a[r0 + t] = W_o att + res in it (fused_decode_ldg_mlp.inl:24-68).
-MQ_DEV void o_publish(float* a_out, int wg, int G, const float* lds, float& res) {
-  int r0, nr;
-  row_range(MQ_H, wg, G, r0, nr);
-  const int t = lane_id();
-  if (t < nr) {
-    res = (lds[LDS_PR + 2 * t] + lds[LDS_PR + 2 * t + 1]) + res;
-    st_coh(a_out + r0 + t, res);
-  }
 }
 
 // ------------------------------------------------------------------------- P4: gate / up
@@ -1886,20 +1860,107 @@ __global__ void __launch_bounds__(MQ_THREADS) mq_op_merge_kernel(MqDecodeParams 
   __shared__ __align__(16) float lds[MQ_LDS_FLOATS];
   attn_merge_head(p.s->part, blockIdx.x, nch, att_out, lds);
 }
-// O projection with residual: a_out = W_o att + x (x bf16, the layer input).
-__global__ void __launch_bounds__(MQ_THREADS) mq_op_o_kernel(MqDecodeParams p, int l,
-                                                              const float* att, const bf16_t* x,
-                                                              float* a_out) {
+// The middle of one whole layer (mq_launch_op_layer): q/k RMSNorm, RoPE, the K/V cache row,
+// attention over [0, pos] and the O projection, split by kv head as in the persistent kernel
+// (workgroup wg serves head wg % 8; the 8 partial O vectors go to s->opart and the MLP kernels add
+// them to the layer input).  Every attention workgroup normalises and rotates its head's q and k
+// itself, so no kernel stands between the projection and the attention.
+// Up to one 224-position block, every workgroup of a head attends over all positions and goes
+// straight on to its O rows (LOCAL); above it, chunks of the positions are attended by
+// mq_op_layer_attn_kernel and merged here by every workgroup of the head.  The separate rope,
+// attention, merge and O kernels this replaces took 3.2 + 5.6 + 3.0 + 4.1 us, each behind the
+// previous one's end: 32.1 -> 22.9 us per layer at position 127 (7 launches -> 4; 5 above one
+// block).
+__global__ void __launch_bounds__(MQ_THREADS) mq_op_layer_attn_kernel(MqDecodeParams p, int l,
+                                                                       int pos, int nch) {
   __shared__ __align__(16) float lds[MQ_LDS_FLOATS];
-  OSet ws;
-  o_load(ws, p.layers[l], blockIdx.x, gridDim.x);
-  int r0, nr;
-  row_range(MQ_H, blockIdx.x, gridDim.x, r0, nr);
-  float res = lane_id() < nr ? bf16_to_f32(x[r0 + lane_id()]) : 0.f;
-  phase_sync(MQ_NOTHING,
-             [&] { wave_copy_coh<MQ_QDIM>(lds + LDS_IN, att); });
-  o_run(ws, p.layers[l], blockIdx.x, gridDim.x, lds);
-  phase_finish([&] { o_publish(a_out, blockIdx.x, gridDim.x, lds, res); });
+  const AttnItem it = attn_item(blockIdx.x, nch, pos + 1);
+  if (!it.active) return;
+  const MqLayerW w = p.layers[l];
+  KvBlock kv;
+  kv_block_load<false>(kv, kv_base(p.kc, p, l, it.h), kv_base(p.vc, p, l, it.h), it.p0,
+                       min(it.p1, it.p0 + MQ_ATT_BLOCK), pos, p.cos);
+  q_operand_clear(lds);
+  phase_sync(MQ_NOTHING, [&] {
+    attn_input_f(p.s->qkv, w.q_norm, w.k_norm, p.cos + (size_t)pos * MQ_D,
+                 p.sin + (size_t)pos * MQ_D, it.h, p.scale_log2, lds);
+  });
+  const bool has_new = pos >= it.p0 && pos < it.p1;
+  attn_core(p, l, it.h, it.p0, it.p1, pos, has_new, kv, lds);
+  attn_write_partial(p.s->part, it.h, it.c, lds);
+  if (has_new && wave_id() == MQ_SYNC_WAVE) attn_cache_row(p, l, it.h, pos, lds);
+}
+template <bool LOCAL>
+__global__ void __launch_bounds__(MQ_THREADS) mq_op_layer_o_kernel(MqDecodeParams p, int l, int pos,
+                                                                    int nch) {
+  __shared__ __align__(16) float lds[MQ_LDS_FLOATS];
+  const int h = blockIdx.x % MQ_GROUPS, j = blockIdx.x / MQ_GROUPS, NG = gridDim.x / MQ_GROUPS;
+  const MqLayerW w = p.layers[l];
+  OPairSet ws;
+  if constexpr (LOCAL) {
+    KvBlock kv;
+    kv_block_load<false>(kv, kv_base(p.kc, p, l, h), kv_base(p.vc, p, l, h), 0, pos + 1, pos, p.cos);
+    opart_load(ws, w, h, j, NG);
+    q_operand_clear(lds);
+    phase_sync(MQ_NOTHING, [&] {
+      attn_input_f(p.s->qkv, w.q_norm, w.k_norm, p.cos + (size_t)pos * MQ_D,
+                   p.sin + (size_t)pos * MQ_D, h, p.scale_log2, lds);
+    });
+    attn_core(p, l, h, 0, pos + 1, pos, true, kv, lds, true);
+    if (j == 0 && wave_id() == MQ_SYNC_WAVE) attn_cache_row(p, l, h, pos, lds);
+  } else {
+    opart_load(ws, w, h, j, NG);
+    attn_merge(p.s->part, h, nch, lds, [&](int jj, int d, float o) { lds[LDS_ATTH + jj * MQ_D + d] = o; });
+    __syncthreads();
+  }
+  opart_run(ws, w, h, j, NG, lds);
+  phase_finish([&] {
+    int r0, nr;
+    row_range(MQ_H, j, NG, r0, nr);
+    for (int t = lane_id(); t < nr; t += 64) st_coh(p.s->opart + h * MQ_H + r0 + t, lds[LDS_PR + t]);
+  });
+}
+// a = x + sum_h opart_h of rows r, r + 1 (r even), in head order
+MQ_DEV float2 op_layer_a2(const MqDecodeParams& p, const bf16_t* x, int r) {
+  float2 o[MQ_NKV];
+#pragma unroll
+  for (int h = 0; h < MQ_NKV; ++h) o[h] = ld_coh2(p.s->opart + h * MQ_H + r);
+  const uint32_t xv = ld32(x + r);
+  float2 a = make_float2(bf16_lo(xv), bf16_hi(xv));
+#pragma unroll
+  for (int h = 0; h < MQ_NKV; ++h) {
+    a.x += o[h].x;
+    a.y += o[h].y;
+  }
+  return a;
+}
+__global__ void __launch_bounds__(MQ_THREADS) mq_op_layer_gateup_kernel(MqDecodeParams p, int l,
+                                                                         const bf16_t* x) {
+  __shared__ __align__(16) float lds[MQ_LDS_FLOATS];
+  GateUpSet ws;
+  gu_load(ws, p.layers[l], blockIdx.x, gridDim.x);
+  reinterpret_cast<float2*>(lds + LDS_IN)[tid()] = op_layer_a2(p, x, 2 * tid());
+  __syncthreads();
+  gu_run(ws, p.layers[l], blockIdx.x, gridDim.x, lds);
+  phase_finish([&] { gu_publish_f(p.s->mlp, blockIdx.x, gridDim.x, lds); });
+}
+__global__ void __launch_bounds__(MQ_THREADS) mq_op_layer_down_kernel(MqDecodeParams p, int l,
+                                                                       const bf16_t* x,
+                                                                       bf16_t* x_out) {
+  __shared__ __align__(16) float lds[MQ_LDS_FLOATS];
+  DownSet ws;
+  down_load(ws, p.layers[l], blockIdx.x, gridDim.x);
+  int r0, nr;                                       // whole row pairs
+  hid_rows(blockIdx.x, gridDim.x, r0, nr);
+  const int t = lane_id();
+  float2 a = make_float2(0.f, 0.f);
+  if (wave_id() == MQ_SYNC_WAVE && t < nr) a = op_layer_a2(p, x, r0 + (t & ~1));
+  float res = t & 1 ? a.y : a.x;
+  phase_sync(MQ_NOTHING, [&] { wave_copy_coh<MQ_I>(lds + LDS_IN, p.s->mlp); });
+  down_run(ws, p.layers[l], blockIdx.x, gridDim.x, lds);
+  phase_finish([&] {
+    down_publish(blockIdx.x, gridDim.x, lds, res, [&](int r, float v) { x_out[r] = f32_to_bf16(v); });
+  });
 }
 // (c) SwiGLU MLP with residual: x_out = bf16(W_d (silu(W_g n) * W_u n) + a), n = RMSNorm(a).
 __global__ void __launch_bounds__(MQ_THREADS) mq_op_gateup_kernel(MqDecodeParams p, int l,
@@ -2947,16 +3008,16 @@ int mq_launch_op_mlp(const MqDecodeParams& p, int layer, const float* a_in, bf16
 
 int mq_launch_op_layer(const MqDecodeParams& p, int layer, const bf16_t* x, int pos,
                        bf16_t* x_out, int grid, hipStream_t stream) {
-  // Scratch use: q_hat -> s->mlp (free until gate/up), attention -> s->att, O output -> s->a.
-  MqScratch* s = p.s;
   const int nch = mq_attn_nchunks(pos + 1, grid);
   mq_op_qkv_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, x);
-  mq_op_rope_kernel<<<MQ_NKV, MQ_THREADS, 0, stream>>>(p, layer, pos, s->mlp);
-  mq_op_attn_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, s->mlp, pos + 1, nch);
-  mq_op_merge_kernel<<<MQ_NKV, MQ_THREADS, 0, stream>>>(p, nch, s->att);
-  mq_op_o_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, s->att, x, s->a);
-  mq_op_gateup_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, s->a);
-  mq_op_down_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, s->a, x_out);
+  if (pos + 1 <= MQ_ATT_BLOCK) {
+    mq_op_layer_o_kernel<true><<<grid, MQ_THREADS, 0, stream>>>(p, layer, pos, 1);
+  } else {
+    mq_op_layer_attn_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, pos, nch);
+    mq_op_layer_o_kernel<false><<<grid, MQ_THREADS, 0, stream>>>(p, layer, pos, nch);
+  }
+  mq_op_layer_gateup_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, x);
+  mq_op_layer_down_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, x, x_out);
   return launch_status();
 }
 

@@ -82,6 +82,35 @@ def test_op_decode_layer_matches_oracle_and_decoder(pair):
     dec.check()
 
 
+# both sides of the one-block (224 positions) / split switch and of a chunk's edge; in the split
+# form the last chunk may hold the new position alone (225, 449), and at 7169 and above every
+# chunk spans more than one 224-position block
+@pytest.mark.parametrize("pos", [0, 1, 222, 223, 224, 225, 447, 448, 449, 1500, 7168, 7300])
+def test_op_decode_layer_attention_split(pos):
+    """mq_op_decode_layer over a random cache against the oracle layer, the written K/V rows
+    included and no other row touched."""
+    from tests.helpers import bf16_ulp, oracle_kv_row
+    dec, orc, _, _ = build_pair(1, 64, 7424, seed=6, norm_jitter=0.1)
+    g = torch.Generator().manual_seed(pos)
+    kc = torch.randn(dec.k_cache.shape, generator=g).to(torch.bfloat16)
+    vc = torch.randn(dec.v_cache.shape, generator=g).to(torch.bfloat16)
+    dec.k_cache.copy_(kc)
+    dec.v_cache.copy_(vc)
+    x = torch.randn(1024, generator=g).to(torch.bfloat16)
+    y = dec.op_decode_layer(0, x.cuda(), pos).float().cpu()
+    orc.k_cache, orc.v_cache = dec.k_cache.float().cpu(), dec.v_cache.float().cpu()
+    for got, own, before in zip((orc.k_cache, orc.v_cache), oracle_kv_row(orc, 0, x.float(), pos),
+                                (kc, vc)):
+        row = got[0, :, pos]
+        assert ((row - own).abs() <= bf16_ulp(own) + 2e-5 * own.abs().amax(-1, keepdim=True)).all()
+        rest = got.clone()
+        rest[0, :, pos] = before[0, :, pos].float()
+        assert torch.equal(rest, before.float())
+    ref = orc.decode_layer(0, x.float(), pos, write_kv=False)
+    assert ((y - ref).abs() <= _bf16_ulp(ref) + 2e-5 * float(ref.abs().max())).all()
+    dec.check()
+
+
 def test_chat_decode_ldg_matches_decoder(pair):
     """chat.py's decode_ldg / decode_ldg_with_logits over caller-owned caches: against the CPU
     oracle directly (teacher-forced, north-star 2e-2 on the logits, greedy tokens wherever the
