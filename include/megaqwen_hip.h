@@ -270,6 +270,10 @@ size_t mq_flash_attn_workspace_bytes(int batch, int heads, int seq_len, int head
 int mq_flash_attn_bhwd(const void* d_q, const void* d_k, const void* d_v, void* d_out,
                        int batch, int heads, int seq_len, int head_dim, int dtype, float scale,
                        void* d_workspace, size_t workspace_bytes, void* stream);
+/* The same without the workspace argument. */
+int mq_flash_attn_bhwd_nows(const void* d_q, const void* d_k, const void* d_v, void* d_out,
+                            int batch, int heads, int seq_len, int head_dim, int dtype,
+                            float scale, void* stream);
 
 #ifdef __cplusplus
 }

@@ -31,7 +31,7 @@ EXPORTED = (
     "mq_decoder_set_host_position", "mq_decoder_set_position", "mq_decoder_set_mode", "mq_decoder_get_mode", "mq_decoder_grid", "mq_decode_step",
     "mq_decode_steps", "mq_debug_decode_step_layers", "mq_debug_decode_step_timing", "mq_decoder_check", "mq_prefill", "mq_prefill_embeds", "mq_prefill_fused", "mq_debug_prefill_layers", "mq_debug_prefill_buffers", "mq_op_qkv_rope", "mq_op_attention", "mq_op_attention_noalloc",
     "mq_op_mlp", "mq_op_decode_layer", "mq_op_lm_head", "mq_flash_attn_workspace_bytes",
-    "mq_flash_attn_bhwd", "mq_exchange_epoch", "mq_exchange_epoch_advance", "mq_exchange_tag",
+    "mq_flash_attn_bhwd", "mq_flash_attn_bhwd_nows", "mq_exchange_epoch", "mq_exchange_epoch_advance", "mq_exchange_tag",
     "mq_exchange_epoch_period", "mq_debug_set_exchange_epoch", "mq_debug_get_exchange_epoch",
 )
 
@@ -104,6 +104,7 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         "mq_op_lm_head": (I, [P, P, P, P, P]),
         "mq_flash_attn_workspace_bytes": (S, [I, I, I, I]),
         "mq_flash_attn_bhwd": (I, [P, P, P, P, I, I, I, I, I, ctypes.c_float, P, S, P]),
+        "mq_flash_attn_bhwd_nows": (I, [P, P, P, P, I, I, I, I, I, ctypes.c_float, P]),
         "mq_exchange_epoch": (U32, [U32, ctypes.c_uint64]),
         "mq_exchange_epoch_advance": (U32, [U32, ctypes.c_uint64]),
         "mq_exchange_tag": (U32, [U32]),

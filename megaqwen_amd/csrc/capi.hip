@@ -608,9 +608,10 @@ size_t mq_flash_attn_workspace_bytes(int batch, int heads, int seq_len, int head
   return mq_flash_attn_workspace(batch * heads, seq_len);
 }
 
-int mq_flash_attn_bhwd(const void* d_q, const void* d_k, const void* d_v, void* d_out,
-                       int batch, int heads, int seq_len, int head_dim, int dtype, float scale,
-                       void* d_workspace, size_t workspace_bytes, void* stream) {
+// Checks shared by the two entry points; *run is false for an empty problem.
+static int check_flash_attn(const void* d_q, const void* d_k, const void* d_v, const void* d_out,
+                            int batch, int heads, int seq_len, int head_dim, int dtype, bool* run) {
+  *run = false;
   if (batch < 0 || heads < 0 || seq_len < 0)
     return fail(MQ_ERR_INVALID_ARG, "negative size (batch %d, heads %d, seq_len %d)", batch,
                 heads, seq_len);
@@ -631,15 +632,40 @@ int mq_flash_attn_bhwd(const void* d_q, const void* d_k, const void* d_v, void* 
   };
   if (overlaps(d_out, d_k) || overlaps(d_out, d_v))
     return fail(MQ_ERR_INVALID_ARG, "out must not overlap k or v");
-  const size_t ws = mq_flash_attn_workspace(batch * heads, seq_len);
-  if (d_workspace == nullptr || workspace_bytes < ws || (reinterpret_cast<uintptr_t>(d_workspace) & 15) != 0)
-    return fail(MQ_ERR_INVALID_ARG, "workspace needs %zu bytes, 16-byte aligned (got %zu)", ws,
-                workspace_bytes);
+  *run = true;
+  return MQ_OK;
+}
+
+static int launch_flash_attn(const void* d_q, const void* d_k, const void* d_v, void* d_out,
+                             int batch, int heads, int seq_len, int dtype, float scale,
+                             void* stream) {
   const float scale_log2 = (float)((double)scale * 1.4426950408889634);
   const int rc = mq_launch_flash_attn_bhwd(d_q, d_k, d_v, d_out, batch * heads, seq_len,
                                            dtype == MQ_DTYPE_F16, scale_log2,
                                            static_cast<hipStream_t>(stream));
   return rc == 0 ? MQ_OK : fail(MQ_ERR_HIP, "launch failed (%s)", hipGetErrorString(hipGetLastError()));
+}
+
+int mq_flash_attn_bhwd(const void* d_q, const void* d_k, const void* d_v, void* d_out,
+                       int batch, int heads, int seq_len, int head_dim, int dtype, float scale,
+                       void* d_workspace, size_t workspace_bytes, void* stream) {
+  bool run;
+  const int rc = check_flash_attn(d_q, d_k, d_v, d_out, batch, heads, seq_len, head_dim, dtype, &run);
+  if (rc != MQ_OK || !run) return rc;
+  const size_t ws = mq_flash_attn_workspace(batch * heads, seq_len);
+  if (d_workspace == nullptr || workspace_bytes < ws || (reinterpret_cast<uintptr_t>(d_workspace) & 15) != 0)
+    return fail(MQ_ERR_INVALID_ARG, "workspace needs %zu bytes, 16-byte aligned (got %zu)", ws,
+                workspace_bytes);
+  return launch_flash_attn(d_q, d_k, d_v, d_out, batch, heads, seq_len, dtype, scale, stream);
+}
+
+int mq_flash_attn_bhwd_nows(const void* d_q, const void* d_k, const void* d_v, void* d_out,
+                            int batch, int heads, int seq_len, int head_dim, int dtype,
+                            float scale, void* stream) {
+  bool run;
+  const int rc = check_flash_attn(d_q, d_k, d_v, d_out, batch, heads, seq_len, head_dim, dtype, &run);
+  if (rc != MQ_OK || !run) return rc;
+  return launch_flash_attn(d_q, d_k, d_v, d_out, batch, heads, seq_len, dtype, scale, stream);
 }
 
 }  // extern "C"

@@ -63,17 +63,18 @@ def flash_attn_bhwd(
     out = torch.empty_like(q)
     if out.numel() == 0:
         return out
-    lib = _lib.load()
     dtype = _lib.MQ_DTYPE_F16 if q.dtype == torch.float16 else _lib.MQ_DTYPE_BF16
-    ws_bytes = lib.mq_flash_attn_workspace_bytes(b, h, t, d)
-    if ws_bytes == 0:
-        _lib.check(_lib.MQ_ERR_INVALID_ARG)
-    # the scratch the C interface asks for (stream-ordered, so the caching allocator may hand the
-    # block out again once the call is queued)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        _lib.check(lib.mq_flash_attn_bhwd(q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                          out.data_ptr(), b, h, t, d, dtype, float(scale),
-                                          ws.data_ptr(), ws_bytes, stream))
+    # a short clip's kernel takes ~5 us, so the call is as fast as this function: the entry point
+    # without a workspace, the raw stream handle, and no device guard when the tensors are on the
+    # current device (13.0 -> 7.6 us per call at 14 heads, T = 99)
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, t, d, dtype, scale)
+    dev = q.get_device()
+    call = _lib.load().mq_flash_attn_bhwd_nows
+    if dev == torch.cuda.current_device():
+        rc = call(*args, torch._C._cuda_getCurrentRawStream(dev))
+    else:
+        with torch.cuda.device(dev):
+            rc = call(*args, torch._C._cuda_getCurrentRawStream(dev))
+    if rc != 0:
+        _lib.check(rc)
     return out

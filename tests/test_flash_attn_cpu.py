@@ -107,5 +107,12 @@ def test_c_abi_rejections():
     assert b"workspace" in lib.mq_last_error()
     assert f(fake, 2 * fake, 3 * fake, 4 * fake, 1, 1, 40, 64, bf, 1.0, None, 1 << 20, None) \
         == _lib.MQ_ERR_INVALID_ARG
+    # the entry point without a workspace makes the same checks
+    n = lib.mq_flash_attn_bhwd_nows
+    assert n(fake, fake, fake, fake, 1, 1, 4, 128, bf, 1.0, None) == _lib.MQ_ERR_INVALID_ARG
+    assert n(None, fake, fake, fake, 1, 1, 4, 64, bf, 1.0, None) == _lib.MQ_ERR_INVALID_ARG
+    assert n(fake, 2 * fake, 3 * fake, 3 * fake + 64, 1, 1, 4, 64, bf, 1.0, None) \
+        == _lib.MQ_ERR_INVALID_ARG
+    assert n(None, None, None, None, 1, 14, 0, 64, bf, 1.0, None) == _lib.MQ_OK
     # empty problems are no-ops (nothing is launched)
     assert f(None, None, None, None, 1, 14, 0, 64, bf, 1.0, None, 0, None) == _lib.MQ_OK
