@@ -238,7 +238,6 @@ int mq_decoder_create(const mq_model_desc* desc, void* k_cache, void* v_cache, v
   memset(&dec->fused, 0, sizeof(dec->fused));
   if (desc->max_prefill_len > 0) mq_fused_bind(&dec->fused, ws + lay.fused, desc->num_layers);
   if (mq_launch_clear_state(p.st, p.x, nullptr) != 0 || clear_fused_tags(dec, nullptr) != 0 ||
-      (dec->pf.cnt != nullptr && mq_launch_zero(dec->pf.cnt, dec->pf.cnt_bytes, nullptr) != 0) ||
       hipStreamSynchronize(nullptr) != hipSuccess) {
     delete dec;
     return fail(MQ_ERR_HIP, "state initialisation failed");
@@ -257,8 +256,7 @@ int mq_decoder_reset(mq_decoder* dec, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (mq_launch_zero(dec->p.kc, dec->kv_bytes, s) != 0 ||
       mq_launch_zero(dec->p.vc, dec->kv_bytes, s) != 0 ||
-      mq_launch_clear_state(dec->p.st, dec->p.x, s) != 0 || clear_fused_tags(dec, s) != 0 ||
-      (dec->pf.cnt != nullptr && mq_launch_zero(dec->pf.cnt, dec->pf.cnt_bytes, s) != 0))
+      mq_launch_clear_state(dec->p.st, dec->p.x, s) != 0 || clear_fused_tags(dec, s) != 0)
     return fail(MQ_ERR_HIP, "reset kernels failed to launch");
   dec->pos = 0;
   return MQ_OK;

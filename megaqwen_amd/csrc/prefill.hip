@@ -8,9 +8,11 @@
 //   q,k = bf16(RoPE(RMSNorm_head(.) * w)); k, v -> KV cache rows    the same GEMM's epilogue
 //   att = bf16(causal GQA softmax(q k^T / sqrt(128)) v)             MFMA flash attention
 //   h   = bf16(bf16(att Wo^T) + h)                                  MFMA GEMM + residual epilogue
-//   xn  = bf16(RMSNorm(h) * w_post)
+//   xn  = bf16(RMSNorm(h) * w_post)                                 row kernel
 //   m   = bf16(silu(bf16(xn Wg^T)) * bf16(xn Wu^T))                 dual MFMA GEMM + SwiGLU
 //   h   = bf16(bf16(m Wd^T) + h)                                    MFMA GEMM + residual epilogue
+// (up to 768 rows the O and down GEMMs leave split-K sums instead, and one row kernel adds them,
+// the residual and the norm that follows)
 // then the last row's final norm (bf16) and the LM-head argmax (fused_prefill_kernels.inl:655-824).
 //
 // GEMMs are C[M,N] = A[M,K] B[N,K]^T ("NT": activations and weights both K-contiguous) on
@@ -112,8 +114,55 @@ __global__ void __launch_bounds__(128) pf_rmsnorm_kernel(const bf16_t* __restric
   reinterpret_cast<uint4*>(y + (size_t)row * MQ_H)[t] = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
+// h += bf16(sum over the splits of a projection's fp32 partials [sk][M][H], in split order), rounded
+// as the residual epilogue does, and, unless w is NULL, y = bf16(RMSNorm(h) * w) of the new row: the
+// residual add of the O and down projections and the norm that follows it in one kernel.
+__global__ void __launch_bounds__(128) pf_sum_norm_kernel(const float* __restrict__ part, int sk,
+                                                          int M, bf16_t* __restrict__ h,
+                                                          const bf16_t* __restrict__ w,
+                                                          bf16_t* __restrict__ y) {
+  __shared__ float red[2];
+  const int row = blockIdx.x, t = threadIdx.x;
+  const float4* src = reinterpret_cast<const float4*>(part + (size_t)row * MQ_H + 8 * t);
+  const size_t stride = (size_t)M * MQ_H / 4;
+  const uint4 hv = reinterpret_cast<const uint4*>(h + (size_t)row * MQ_H)[t];
+  const uint4 wq = w != nullptr ? reinterpret_cast<const uint4*>(w)[t] : make_uint4(0, 0, 0, 0);
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int z = 0; z < sk; ++z) {
+    const float4 a = src[z * stride], b = src[z * stride + 1];
+    s[0] += a.x; s[1] += a.y; s[2] += a.z; s[3] += a.w;
+    s[4] += b.x; s[5] += b.y; s[6] += b.z; s[7] += b.w;
+  }
+  float v[8];
+  unpack8(hv, v);
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    v[e] = round_bf16(round_bf16(s[e]) + v[e]);
+    ss = fmaf(v[e], v[e], ss);
+  }
+  uint32_t o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    o[e] = (uint32_t)f32_to_bf16(v[2 * e]) | ((uint32_t)f32_to_bf16(v[2 * e + 1]) << 16);
+  reinterpret_cast<uint4*>(h + (size_t)row * MQ_H)[t] = make_uint4(o[0], o[1], o[2], o[3]);
+  if (w == nullptr) return;
+  ss = wave_sum(ss);
+  if ((t & 63) == 0) red[t >> 6] = ss;
+  __syncthreads();
+  const float r = rsqrtf((red[0] + red[1]) * (1.0f / MQ_H) + MQ_EPS);
+  float wv[8];
+  unpack8(wq, wv);
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    o[e] = (uint32_t)f32_to_bf16(v[2 * e] * r * wv[2 * e]) |
+           ((uint32_t)f32_to_bf16(v[2 * e + 1] * r * wv[2 * e + 1]) << 16);
+  reinterpret_cast<uint4*>(y + (size_t)row * MQ_H)[t] = make_uint4(o[0], o[1], o[2], o[3]);
+}
+
 // ------------------------------------------------------------------------------ GEMM
-enum { EPI_STORE = 0, EPI_RESID = 1, EPI_SWIGLU = 2, EPI_QKV = 3 };
+enum { EPI_STORE = 0, EPI_RESID = 1, EPI_SWIGLU = 2, EPI_QKV = 3, EPI_PART = 4 };
 
 struct GemmArgs {
   const bf16_t* A;   // [M, K]
@@ -142,13 +191,8 @@ struct GemmArgs {
   bf16_t* Kt;
   int max_seq;
   int M, N, K;
-  // split-K (gridDim.z = sk > 1): every split writes its fp32 partial tile to `part` with
-  // device-coherent stores; the last split of a tile to arrive (counter `cnt[tile]`, reset by
-  // it to 0) sums the sk partials in split order and runs the epilogue, so the result does not
-  // depend on which split finishes last
-  int sk;
-  float* part;       // [tiles][sk][elements per thread][threads]
-  uint32_t* cnt;     // [tiles], 0 between uses
+  int sk;            // K splits (gridDim.z); above 1 only with EPI_PART
+  float* part;       // EPI_PART: fp32 sums of each split, [sk][M][N]
 };
 
 #define GEMM_BK 64           // K per step of 64- and 128-row tiles (32-row tiles: 128)
@@ -413,55 +457,21 @@ __global__ void __launch_bounds__(256) pf_gemm_kernel(GemmArgs g) {
     for (int j = 0; j < 16; ++j) acc[0][0][0][j] += red[(wn * 16 + j) * 64 + lane];
   }
 
-  if (g.sk > 1) {
-    // split-K fixup (the waves left after the K-group merge: 128 or 256 threads)
-    constexpr int E = NB * MB * NBK * 16;
-    constexpr int NT = KG == 2 ? 128 : 256;
-    __shared__ uint32_t is_last;
-    const int tile = blockIdx.y * gridDim.x + blockIdx.x;
-    float* mine = g.part + ((size_t)tile * g.sk + blockIdx.z) * E * NT + t;
-    {
-      int e = 0;
+  if constexpr (EPI == EPI_PART) {
+    // this split's fp32 sums, [split][M][N]; pf_sum_norm_kernel adds them up
+    float* dst = g.part + (size_t)blockIdx.z * g.M * g.N;
 #pragma unroll
-      for (int b = 0; b < NB; ++b)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
+      for (int nb = 0; nb < NBK; ++nb) {
+        const int col = n_base + wn * WN + nb * 32 + (lane & 31);
 #pragma unroll
-          for (int nb = 0; nb < NBK; ++nb)
-#pragma unroll
-            for (int j = 0; j < 16; ++j, ++e) st_coh(mine + (size_t)e * NT, acc[b][mb][nb][j]);
-    }
-    wait_all_memory();            // this thread's partial is stored ...
-    __syncthreads();              // ... and every other thread's
-    if (t == 0) {
-      const uint32_t prev = __hip_atomic_fetch_add(g.cnt + tile, 1u, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-      is_last = prev + 1 == (uint32_t)g.sk;
-      if (is_last) __hip_atomic_store(g.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (!is_last) return;
-    const float* base = g.part + (size_t)tile * g.sk * E * NT + t;
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < NBK; ++nb)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) acc[b][mb][nb][j] = 0.f;
-    for (int sp = 0; sp < g.sk; ++sp) {
-      const float* src = base + (size_t)sp * E * NT;
-      int e = 0;
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-          for (int nb = 0; nb < NBK; ++nb)
-#pragma unroll
-            for (int j = 0; j < 16; ++j, ++e) acc[b][mb][nb][j] += ld_coh(src + (size_t)e * NT);
-    }
+        for (int j = 0; j < 16; ++j) {
+          const int row = m_base + wm * WM + mb * 32 + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
+          if (row < g.M) dst[(size_t)row * g.N + col] = acc[0][mb][nb][j];
+        }
+      }
+    return;
   }
 
   if constexpr (EPI == EPI_QKV) {
@@ -775,16 +785,14 @@ static size_t pf_align(size_t v) { return (v + 255) / 256 * 256; }
 // 32-key tiles per kv head of the K / V^T operand copies
 static int pf_tiles(int max_n) { return (max_n + 31) / 32; }
 
-static void pf_split_sizes(int max_n, size_t& part_bytes, size_t& tiles);
+static size_t pf_part_bytes(int max_n);
 
 size_t mq_prefill_workspace_bytes(int max_n) {
   if (max_n <= 0) return 0;
   const size_t n = (size_t)max_n;
-  size_t part, tiles;
-  pf_split_sizes(max_n, part, tiles);
   return pf_align(n * MQ_H * 2) * 2 + pf_align(n * MQ_QKV * 2) + pf_align(n * MQ_QDIM * 2) +
          pf_align(n * MQ_I * 2) + 2 * pf_align((size_t)MQ_NKV * pf_tiles(max_n) * 4096 * 2) +
-         pf_align(part) + pf_align(tiles * 4);
+         pf_align(pf_part_bytes(max_n));
 }
 
 void mq_prefill_bind(MqPrefillBuffers* b, char* base, int max_n) {
@@ -794,8 +802,6 @@ void mq_prefill_bind(MqPrefillBuffers* b, char* base, int max_n) {
     b->kt = nullptr;
     b->ntiles = 0;
     b->part = nullptr;
-    b->cnt = nullptr;
-    b->cnt_bytes = 0;
     return;
   }
   const size_t n = (size_t)max_n;
@@ -810,12 +816,7 @@ void mq_prefill_bind(MqPrefillBuffers* b, char* base, int max_n) {
   c += pf_align((size_t)MQ_NKV * b->ntiles * 4096 * 2);
   b->kt = reinterpret_cast<bf16_t*>(c);
   c += pf_align((size_t)MQ_NKV * b->ntiles * 4096 * 2);
-  size_t part, tiles;
-  pf_split_sizes(max_n, part, tiles);
   b->part = reinterpret_cast<float*>(c);
-  c += pf_align(part);
-  b->cnt = reinterpret_cast<uint32_t*>(c);
-  b->cnt_bytes = pf_align(tiles * 4);
 }
 
 // K must be a multiple of 512 and N of 128 (every Qwen3-0.6B projection is).
@@ -825,60 +826,74 @@ static_assert(MQ_H % 512 == 0 && MQ_QDIM % 512 == 0 && MQ_I % 512 == 0, "GEMM K 
 // (two per CU; large M); for the N = 1024 GEMMs (O, down) 128 x 64 when that gives >= 512
 // (M >= 4096: the 64 x 64 tiles' waves wait on LDS issue, three LDS instructions per MFMA;
 // 4096-token prefill 9.6 -> 9.4 ms with the 4-stage ring above); otherwise 64 x 64, or 32 x 64
-// when even 64-row tiles would leave CUs idle (M <= 1024).
-//
-// Tile and split plan of one GEMM (shared by the launcher and the workspace sizing).
+// when even 64-row tiles would leave CUs idle (M <= 960; only above 768, part_plan below).
 struct GemmPlan {
-  int bm, bn, gx, gy, sk, nb;
+  int bm, bn, gx, gy;
 };
-// Smallest split of K that gives >= 480 workgroups (about two per CU), else the largest
-// allowed: a split's K must hold a whole ring of steps (BK x S).
-static int pick_sk(int tiles, int K, int bk, int stages) {
-  const int cands[] = {1, 2, 3, 4, 6, 8};
-  int best = 1;
-  for (int sk : cands) {
-    if (K % sk != 0 || (K / sk) % (bk * stages) != 0) continue;
-    best = sk;
-    if (tiles * sk >= 480) break;
-  }
-  return best;
-}
 template <int EPI>
-static GemmPlan gemm_plan(int M, int N, int K) {
+static GemmPlan gemm_plan(int M, int N) {
   const int mt128 = (M + 127) / 128;
-  GemmPlan pl{64, 64, N / 64, (M + 63) / 64, 1, EPI == EPI_SWIGLU ? 2 : 1};
+  GemmPlan pl{64, 64, N / 64, (M + 63) / 64};
   if constexpr (EPI == EPI_SWIGLU) {
-    if ((N / 64) * mt128 >= 512) pl = GemmPlan{128, 64, N / 64, mt128, 1, 2};
+    if ((N / 64) * mt128 >= 512) pl = GemmPlan{128, 64, N / 64, mt128};
   } else if constexpr (EPI == EPI_QKV) {
     // one 128-column head per tile
-    if ((N / 128) * mt128 >= 512) pl = GemmPlan{128, 128, N / 128, mt128, 1, 1};
-    else pl = GemmPlan{64, 128, N / 128, (M + 63) / 64, 1, 1};
+    if ((N / 128) * mt128 >= 512) pl = GemmPlan{128, 128, N / 128, mt128};
+    else pl = GemmPlan{64, 128, N / 128, (M + 63) / 64};
   } else {
-    if ((N / 128) * mt128 >= 512) pl = GemmPlan{128, 128, N / 128, mt128, 1, 1};
-    else if ((N / 64) * mt128 >= 512) pl = GemmPlan{128, 64, N / 64, mt128, 1, 1};
-    else if ((N / 64) * ((M + 63) / 64) < 256) pl = GemmPlan{32, 64, N / 64, (M + 31) / 32, 1, 1};
+    if ((N / 128) * mt128 >= 512) pl = GemmPlan{128, 128, N / 128, mt128};
+    else if ((N / 64) * mt128 >= 512) pl = GemmPlan{128, 64, N / 64, mt128};
+    else if ((N / 64) * ((M + 63) / 64) < 256) pl = GemmPlan{32, 64, N / 64, (M + 31) / 32};
   }
-  // K is split only for the 32 x 64 tiles of short prompts (fewer than 128 tiles, so at most
-  // half the CUs busy): there a split's partial is 8 KB and the fixup costs less than the
-  // longer K loop it removes (O and down at 16 tokens: 11.8 -> 9.5-10 us).  Larger tiles pay
-  // more for the partial round trip than they save (q|k|v and gate|up at 16 tokens 12-12.4 ->
-  // 12.9-13.5 us with 4 splits; every GEMM at 512 tokens slower with 2 splits, e.g. gate|up
-  // 18.0 -> 23.9 us).
-  if (pl.bm == 32 && pl.gx * pl.gy < 128) pl.sk = pick_sk(pl.gx * pl.gy, K, 128, GEMM_STAGES);
   return pl;
 }
-// fp32 partial bytes of a plan (0 without a split)
-static size_t plan_part_bytes(const GemmPlan& pl) {
-  return pl.sk > 1 ? (size_t)pl.gx * pl.gy * pl.sk * pl.bm * pl.bn * pl.nb * 4 : 0;
+
+// The N = 1024 projections (O, down) of up to 768 rows: K split over workgroups, each split's fp32
+// sums to memory, added up by the kernel that makes the following norm (pf_sum_norm_kernel).  64-row
+// tiles then fill the CUs, and a CU loads half to three quarters of the bytes the 32 x 64 tiles of
+// the residual epilogue need, whose loads bound them; the sums cost 4 KB per row and split once
+// out and in.  Per layer, O + down, residual epilogue -> split (us, one card): 32 rows -4.5, 128
+// -5.2, 256 -5.5, 384 -2.3, 512 -1.1, 640 -4.9, 768 -4.5; at 1024 rows, where 64 x 64 tiles alone
+// fill the CUs, +1.9.
+struct PartPlan {
+  int bn, sk;        // tile columns and splits; sk 0: residual epilogue
+};
+static PartPlan part_plan(int M) {
+  if (M <= 256) return PartPlan{64, 4};
+  if (M <= 512) return PartPlan{64, 2};
+  if (M <= 768) return PartPlan{128, 2};
+  return PartPlan{64, 0};
+}
+static_assert(MQ_QDIM % (4 * GEMM_BK * GEMM_STAGES) == 0 && MQ_I % (4 * GEMM_BK * GEMM_STAGES) == 0,
+              "every split is a whole number of register-ring rounds");
+// Starts the split products of a projection into b.part and returns the split count, or 0.
+static int gemm_part(GemmArgs g, const MqPrefillBuffers& b, hipStream_t s) {
+  const PartPlan pl = part_plan(g.M);
+  if (pl.sk == 0) return 0;
+  g.sk = pl.sk;
+  g.part = b.part;
+  const dim3 grid(g.N / pl.bn, (g.M + 63) / 64, pl.sk);
+  if (pl.bn == 128) pf_gemm_kernel<EPI_PART, 64, 128><<<grid, 256, 0, s>>>(g);
+  else pf_gemm_kernel<EPI_PART, 64, 64><<<grid, 256, 0, s>>>(g);
+  return pl.sk;
+}
+// Bytes of the split sums over every prompt length up to max_n.
+static size_t pf_part_bytes(int max_n) {
+  const int top[] = {256, 512, 768};                // the longest prompt of each plan
+  size_t bytes = 0;
+  for (int m : top) {
+    const int n = m < max_n ? m : max_n;
+    const size_t v = (size_t)part_plan(n).sk * n * MQ_H * sizeof(float);
+    bytes = bytes > v ? bytes : v;
+  }
+  return bytes;
 }
 
 template <int EPI>
-static void gemm(GemmArgs g, const MqPrefillBuffers& b, hipStream_t s) {
-  const GemmPlan pl = gemm_plan<EPI>(g.M, g.N, g.K);
-  g.sk = pl.sk;
-  g.part = b.part;
-  g.cnt = b.cnt;
-  const dim3 grid(pl.gx, pl.gy, pl.sk);
+static void gemm(GemmArgs g, hipStream_t s) {
+  const GemmPlan pl = gemm_plan<EPI>(g.M, g.N);
+  g.sk = 1;
+  const dim3 grid(pl.gx, pl.gy);
   if (pl.bm == 128 && pl.bn == 64) {
     if constexpr (EPI != EPI_QKV) pf_gemm_kernel<EPI, 128, 64><<<grid, 256, 0, s>>>(g);
   } else if (pl.bm == 128) {
@@ -893,27 +908,6 @@ static void gemm(GemmArgs g, const MqPrefillBuffers& b, hipStream_t s) {
   }
 }
 
-// Largest split-K partial area and tile count over every prompt length up to max_n.
-static void pf_split_sizes(int max_n, size_t& part_bytes, size_t& tiles) {
-  part_bytes = 0;
-  tiles = 0;
-  // plans change with the number of 32-row tiles: every multiple of 32 and, behind the last one,
-  // max_n itself
-  for (int m = 32;; m += 32) {
-    const int mm = m > max_n ? max_n : m;
-    const GemmPlan ps[] = {gemm_plan<EPI_QKV>(mm, MQ_QKV, MQ_H),
-                           gemm_plan<EPI_RESID>(mm, MQ_H, MQ_QDIM),
-                           gemm_plan<EPI_SWIGLU>(mm, MQ_I, MQ_H),
-                           gemm_plan<EPI_RESID>(mm, MQ_H, MQ_I)};
-    for (const GemmPlan& pl : ps) {
-      part_bytes = part_bytes > plan_part_bytes(pl) ? part_bytes : plan_part_bytes(pl);
-      const size_t t = (size_t)pl.gx * pl.gy;
-      tiles = tiles > t ? tiles : t;
-    }
-    if (mm == max_n) break;
-  }
-}
-
 int mq_launch_prefill(const MqDecodeParams& p, const MqLayerW* hl, const MqPrefillBuffers& b,
                       const int32_t* tokens, int n, int32_t* tok_out, float* logits, int grid,
                       hipStream_t stream, const bf16_t* patch, int patch_start, int patch_len,
@@ -924,9 +918,10 @@ int mq_launch_prefill(const MqDecodeParams& p, const MqLayerW* hl, const MqPrefi
   if (patch == nullptr) patch_len = 0;
   pf_embed_kernel<<<n, 128, 0, stream>>>(p.embed, tokens, b.h, patch, patch_start, patch_len,
                                          p.vocab, &p.st->sync.err.v);
+  bool normed = false;         // b.xn already holds this layer's normalised input
   for (int l = 0; l < p.num_layers; ++l) {
     const MqLayerW& w = hl[l];
-    pf_rmsnorm_kernel<<<n, 128, 0, stream>>>(b.h, w.in_ln, b.xn);
+    if (!normed) pf_rmsnorm_kernel<<<n, 128, 0, stream>>>(b.h, w.in_ln, b.xn);
     GemmArgs g{};
     g.A = b.xn; g.lda = MQ_H;
     g.B0 = w.wq; g.B1 = w.wk; g.B2 = w.wv; g.n0 = MQ_QDIM; g.n1 = MQ_QDIM + MQ_KVDIM;
@@ -936,25 +931,36 @@ int mq_launch_prefill(const MqDecodeParams& p, const MqLayerW* hl, const MqPrefi
     g.kcl = p.kc + (size_t)l * MQ_NKV * p.max_seq * MQ_D;
     g.vcl = p.vc + (size_t)l * MQ_NKV * p.max_seq * MQ_D;
     g.Kt = b.kt;
-    gemm<EPI_QKV>(g, b, stream);
+    gemm<EPI_QKV>(g, stream);
     pf_attn_kernel<<<dim3(MQ_NQ, (n + 31) / 32), 64 * ATT_SPLIT, 0, stream>>>(
         p, l, b.qkv, b.kt, b.vt, b.ntiles, b.att, n);
     g = GemmArgs{};
     g.A = b.att; g.lda = MQ_QDIM;
     g.B0 = g.B1 = g.B2 = w.wo; g.n0 = g.n1 = MQ_H;
     g.C = b.h; g.ldc = MQ_H; g.R = b.h; g.ldr = MQ_H; g.M = n; g.N = MQ_H; g.K = MQ_QDIM;
-    gemm<EPI_RESID>(g, b, stream);
-    pf_rmsnorm_kernel<<<n, 128, 0, stream>>>(b.h, w.post_ln, b.xn);
+    if (const int sk = gemm_part(g, b, stream)) {
+      pf_sum_norm_kernel<<<n, 128, 0, stream>>>(b.part, sk, n, b.h, w.post_ln, b.xn);
+    } else {
+      gemm<EPI_RESID>(g, stream);
+      pf_rmsnorm_kernel<<<n, 128, 0, stream>>>(b.h, w.post_ln, b.xn);
+    }
     g = GemmArgs{};
     g.A = b.xn; g.lda = MQ_H;
     g.B0 = g.B1 = g.B2 = w.wg; g.n0 = g.n1 = MQ_I; g.Bu = w.wu;
     g.C = b.m; g.ldc = MQ_I; g.M = n; g.N = MQ_I; g.K = MQ_H;
-    gemm<EPI_SWIGLU>(g, b, stream);
+    gemm<EPI_SWIGLU>(g, stream);
     g = GemmArgs{};
     g.A = b.m; g.lda = MQ_I;
     g.B0 = g.B1 = g.B2 = w.wd; g.n0 = g.n1 = MQ_H;
     g.C = b.h; g.ldc = MQ_H; g.R = b.h; g.ldr = MQ_H; g.M = n; g.N = MQ_H; g.K = MQ_I;
-    gemm<EPI_RESID>(g, b, stream);
+    normed = false;
+    if (const int sk = gemm_part(g, b, stream)) {
+      // with the next layer's input norm
+      normed = l + 1 < p.num_layers;
+      pf_sum_norm_kernel<<<n, 128, 0, stream>>>(b.part, sk, n, b.h, normed ? hl[l + 1].in_ln : nullptr, b.xn);
+    } else {
+      gemm<EPI_RESID>(g, stream);
+    }
     if (trace != nullptr &&
         hipMemcpyAsync(trace + (size_t)l * n * MQ_H, b.h, (size_t)n * MQ_H * sizeof(bf16_t),
                        hipMemcpyDeviceToDevice, stream) != hipSuccess)

@@ -277,3 +277,30 @@ def test_prefill_of_exactly_max_prefill_len(small, n):
         assert torch.equal(tight.k_cache[:, :, :n], dec.k_cache[:, :, :n])
         assert torch.equal(tight.v_cache[:, :, :n], dec.v_cache[:, :, :n])
     dec.reset()
+
+
+@pytest.fixture(scope="module")
+def mid():
+    return build_pair(2, 4096, 840, seed=5, norm_jitter=0.1, max_prefill=832)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 256, 257, 512, 513, 768, 769, 832])
+def test_prefill_projection_splits(mid, n):
+    """Both sides of every switch of the O and down projections' K split (up to 256 rows, 512, 768,
+    the residual epilogue above) and partial 64-row tiles, against the oracle: the last row's
+    logits, and every row of layer 1's K and V, which all come from layer 0's projections."""
+    dec, orc, sp, _ = mid
+    toks = make_tokens(n, sp["vocab_size"], seed=100 + n)
+    dec.reset()
+    orc.reset()
+    tok, lg = dec.prefill_step_with_logits(toks)
+    _, olg = orc.prefill(toks)
+    err = float((lg.cpu() - olg).abs().max())
+    assert err <= T.PREFILL_2L, err
+    if top2_margin(olg) > 2 * err:
+        assert tok == int(torch.argmax(olg))
+    for got, ref in ((dec.k_cache, orc.k_cache), (dec.v_cache, orc.v_cache)):
+        a, b = got[1, :, :n].float().cpu(), ref[1, :, :n]
+        # layer 1's rows come from layer 0's output: bf16 flips of single activations, not tiles
+        assert float((a - b).norm() / b.norm()) < 1e-2
+        assert float((a - b).abs().amax() / b.abs().amax()) < 5e-2
