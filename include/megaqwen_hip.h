@@ -246,7 +246,8 @@ int mq_op_mlp(mq_decoder* dec, int layer, const float* d_a, void* d_x_out_bf16, 
 /* One whole decoder layer at position `pos` (generate.py:78-110 decode_layer): bf16 hidden in ->
  * bf16 hidden out, writing K/V cache row `pos` of `layer` and attending over rows [0, pos].
  * Uses the decoder's workspace; does not change the decode position.  Input and output must
- * not alias. */
+ * not be the same buffer (MQ_ERR_INVALID_ARG); ranges that overlap otherwise give the result of
+ * separate ones. */
 int mq_op_decode_layer(mq_decoder* dec, int layer, const void* d_x_bf16, int pos,
                        void* d_x_out_bf16, void* stream);
 /* (d) final RMSNorm + LM head + argmax of a bf16 hidden state (fused_decode_ldg_lm.inl:6-163);

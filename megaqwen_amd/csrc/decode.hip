@@ -1934,6 +1934,9 @@ MQ_DEV float2 op_layer_a2(const MqDecodeParams& p, const bf16_t* x, int r) {
   }
   return a;
 }
+// a = x + O output of every row, the MLP on it, and a itself to s->a (each workgroup its rows of the
+// down projection) as that projection's residual: no kernel that writes the layer output reads x,
+// so the two may overlap.
 __global__ void __launch_bounds__(MQ_THREADS) mq_op_layer_gateup_kernel(MqDecodeParams p, int l,
                                                                          const bf16_t* x) {
   __shared__ __align__(16) float lds[MQ_LDS_FLOATS];
@@ -1941,26 +1944,11 @@ __global__ void __launch_bounds__(MQ_THREADS) mq_op_layer_gateup_kernel(MqDecode
   gu_load(ws, p.layers[l], blockIdx.x, gridDim.x);
   reinterpret_cast<float2*>(lds + LDS_IN)[tid()] = op_layer_a2(p, x, 2 * tid());
   __syncthreads();
+  int r0, nr;
+  hid_rows(blockIdx.x, gridDim.x, r0, nr);
+  if (tid() < nr) st_coh(p.s->a + r0 + tid(), lds[LDS_IN + r0 + tid()]);
   gu_run(ws, p.layers[l], blockIdx.x, gridDim.x, lds);
   phase_finish([&] { gu_publish_f(p.s->mlp, blockIdx.x, gridDim.x, lds); });
-}
-__global__ void __launch_bounds__(MQ_THREADS) mq_op_layer_down_kernel(MqDecodeParams p, int l,
-                                                                       const bf16_t* x,
-                                                                       bf16_t* x_out) {
-  __shared__ __align__(16) float lds[MQ_LDS_FLOATS];
-  DownSet ws;
-  down_load(ws, p.layers[l], blockIdx.x, gridDim.x);
-  int r0, nr;                                       // whole row pairs
-  hid_rows(blockIdx.x, gridDim.x, r0, nr);
-  const int t = lane_id();
-  float2 a = make_float2(0.f, 0.f);
-  if (wave_id() == MQ_SYNC_WAVE && t < nr) a = op_layer_a2(p, x, r0 + (t & ~1));
-  float res = t & 1 ? a.y : a.x;
-  phase_sync(MQ_NOTHING, [&] { wave_copy_coh<MQ_I>(lds + LDS_IN, p.s->mlp); });
-  down_run(ws, p.layers[l], blockIdx.x, gridDim.x, lds);
-  phase_finish([&] {
-    down_publish(blockIdx.x, gridDim.x, lds, res, [&](int r, float v) { x_out[r] = f32_to_bf16(v); });
-  });
 }
 // (c) SwiGLU MLP with residual: x_out = bf16(W_d (silu(W_g n) * W_u n) + a), n = RMSNorm(a).
 __global__ void __launch_bounds__(MQ_THREADS) mq_op_gateup_kernel(MqDecodeParams p, int l,
@@ -3031,7 +3019,7 @@ int mq_launch_op_layer(const MqDecodeParams& p, int layer, const bf16_t* x, int 
     mq_op_layer_o_kernel<false><<<grid, MQ_THREADS, 0, stream>>>(p, layer, pos, nch);
   }
   mq_op_layer_gateup_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, x);
-  mq_op_layer_down_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, x, x_out);
+  mq_op_down_kernel<<<grid, MQ_THREADS, 0, stream>>>(p, layer, p.s->a, x_out);
   return launch_status();
 }
 

@@ -31,6 +31,7 @@ struct MqLayerW {
 struct MqScratch {
   float qkv[MQ_QKV];           // raw q | k | v projections (before q/k RMSNorm and RoPE)
   float opart[MQ_NKV * MQ_H];  // O projection restricted to each kv head's query heads (op_layer)
+  float a[MQ_H];               // residual stream after attention: W_o att + x (op_layer)
   float mlp[MQ_I];             // silu(gate) * up
   float part[MQ_NKV * MQ_MAX_CHUNKS * MQ_GQA * MQ_PART_STRIDE];  // attention split-K partials
 };

@@ -111,6 +111,25 @@ def test_op_decode_layer_attention_split(pos):
     dec.check()
 
 
+@pytest.mark.parametrize("pos", [100, 240])
+@pytest.mark.parametrize("shift", [-1016, -512, -8, 8, 512, 1016])
+def test_op_decode_layer_overlapping_ranges(pair, pos, shift):
+    """Input and output ranges that overlap without being equal give the bits of separate ones
+    (the output is written by one kernel, and that kernel must not read the input)."""
+    dec, _, _, _ = pair
+    g = torch.Generator(device="cuda").manual_seed(pos)
+    x = torch.randn(1024, generator=g, device="cuda").to(torch.bfloat16)
+    want = dec.op_decode_layer(0, x, pos)
+    for _ in range(3):
+        buf = torch.zeros(3 * 1024, dtype=torch.bfloat16, device="cuda")
+        src, dst = buf[1024:2048], buf[1024 + shift:2048 + shift]
+        src.copy_(x)
+        got = dec.op_decode_layer(0, src, pos, x_out=dst)
+        assert got.data_ptr() == dst.data_ptr()
+        assert torch.equal(got, want)
+    dec.check()
+
+
 def test_chat_decode_ldg_matches_decoder(pair):
     """chat.py's decode_ldg / decode_ldg_with_logits over caller-owned caches: against the CPU
     oracle directly (teacher-forced, north-star 2e-2 on the logits, greedy tokens wherever the
