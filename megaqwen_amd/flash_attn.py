@@ -67,7 +67,8 @@ def flash_attn_bhwd(
     # a short clip's kernel takes ~5 us, so the call is as fast as this function: the entry point
     # without a workspace, the raw stream handle, and no device guard when the tensors are on the
     # current device (13.0 -> 8.2 us per call at 14 heads, T = 99)
-    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, t, d, dtype, scale)
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, t, d, dtype,
+            float(scale))
     dev = q.get_device()
     call = _lib.load().mq_flash_attn_bhwd_nows
     if dev == torch.cuda.current_device():

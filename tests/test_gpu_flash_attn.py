@@ -64,6 +64,15 @@ def test_batches_heads_scale_and_strided_inputs():
     _check(out.cpu(), q.contiguous(), k.contiguous(), v.contiguous(), scale=0.37)
 
 
+@pytest.mark.parametrize("scale", ["0.25", np.float32(0.25), torch.tensor(0.25)])
+def test_scale_is_anything_float_takes(scale):
+    """`scale` goes through float(): number-like objects and numeric strings alike."""
+    q, k, v = (x.cuda() for x in _inputs((1, 2, 40, 64), torch.bfloat16, seed=6))
+    assert torch.equal(_fa()(q, k, v, scale=scale), _fa()(q, k, v, scale=0.25))
+    with pytest.raises(ValueError):
+        _fa()(q, k, v, scale="a quarter")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_peaked_softmax(dtype):
     """Scores spanning hundreds (inputs of std 6): the running max moves often and most weights
