@@ -856,35 +856,37 @@ static GemmPlan gemm_plan(int M, int N) {
 // -5.2, 256 -5.5, 384 -2.3, 512 -1.1, 640 -4.9, 768 -4.5; at 1024 rows, where 64 x 64 tiles alone
 // fill the CUs, +1.9.
 struct PartPlan {
-  int bn, sk;        // tile columns and splits; sk 0: residual epilogue
+  int rows;          // the longest prompt the plan serves
+  int bn, sk;        // tile columns and splits
 };
-static PartPlan part_plan(int M) {
-  if (M <= 256) return PartPlan{64, 4};
-  if (M <= 512) return PartPlan{64, 2};
-  if (M <= 768) return PartPlan{128, 2};
-  return PartPlan{64, 0};
-}
+static constexpr PartPlan kPartPlans[] = {{256, 64, 4}, {512, 64, 2}, {768, 128, 2}};
 static_assert(MQ_QDIM % (4 * GEMM_BK * GEMM_STAGES) == 0 && MQ_I % (4 * GEMM_BK * GEMM_STAGES) == 0,
               "every split is a whole number of register-ring rounds");
+// Plan of a prompt of M rows, or nullptr for the residual epilogue.
+static const PartPlan* part_plan(int M) {
+  for (const PartPlan& pl : kPartPlans)
+    if (M <= pl.rows) return &pl;
+  return nullptr;
+}
 // Starts the split products of a projection into b.part and returns the split count, or 0.
 static int gemm_part(GemmArgs g, const MqPrefillBuffers& b, hipStream_t s) {
-  const PartPlan pl = part_plan(g.M);
-  if (pl.sk == 0) return 0;
-  g.sk = pl.sk;
+  const PartPlan* pl = part_plan(g.M);
+  if (pl == nullptr) return 0;
+  g.sk = pl->sk;
   g.part = b.part;
-  const dim3 grid(g.N / pl.bn, (g.M + 63) / 64, pl.sk);
-  if (pl.bn == 128) pf_gemm_kernel<EPI_PART, 64, 128><<<grid, 256, 0, s>>>(g);
+  const dim3 grid(g.N / pl->bn, (g.M + 63) / 64, pl->sk);
+  if (pl->bn == 128) pf_gemm_kernel<EPI_PART, 64, 128><<<grid, 256, 0, s>>>(g);
   else pf_gemm_kernel<EPI_PART, 64, 64><<<grid, 256, 0, s>>>(g);
-  return pl.sk;
+  return pl->sk;
 }
-// Bytes of the split sums over every prompt length up to max_n.
+// Bytes of the split sums over every prompt length up to max_n: each plan's longest prompt.
 static size_t pf_part_bytes(int max_n) {
-  const int top[] = {256, 512, 768};                // the longest prompt of each plan
   size_t bytes = 0;
-  for (int m : top) {
-    const int n = m < max_n ? m : max_n;
-    const size_t v = (size_t)part_plan(n).sk * n * MQ_H * sizeof(float);
+  for (const PartPlan& pl : kPartPlans) {
+    const int n = pl.rows < max_n ? pl.rows : max_n;
+    const size_t v = (size_t)pl.sk * n * MQ_H * sizeof(float);
     bytes = bytes > v ? bytes : v;
+    if (pl.rows >= max_n) break;      // no longer prompt, so no further plan
   }
   return bytes;
 }

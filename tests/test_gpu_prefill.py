@@ -258,30 +258,48 @@ def test_prefill_out_of_vocab_id_sets_device_error(small):
     dec.check()
 
 
-@pytest.mark.parametrize("n", [33, 65, 90, 107, 131, 164, 224])
-def test_prefill_of_exactly_max_prefill_len(small, n):
-    """A decoder whose max_prefill_len is the prompt length itself (also off the 32-row tile
-    grid, where the split-K workspace must be sized for the last, partial tile) gives the logits
-    and cache rows of one with room to spare, bit for bit."""
-    dec, _, sp, w = small
+@pytest.fixture(scope="module")
+def mid():
+    return build_pair(2, 4096, 840, seed=5, norm_jitter=0.1, max_prefill=832)
+
+
+@pytest.mark.parametrize("n", [1, 33, 65, 90, 107, 131, 164, 224, 256, 257, 300, 513, 700, 768,
+                               769])
+def test_prefill_of_exactly_max_prefill_len(mid, n):
+    """A decoder whose max_prefill_len is the prompt length itself, in every plan of the O and down
+    projections' K split and off the tile grid, gives the logits and cache rows of one with room to
+    spare, bit for bit, and its split sums, the last of its prefill buffers, end where the buffers
+    do: the fused prefill's area behind them keeps a pattern."""
+    import ctypes
+    from megaqwen_amd import _lib
     from megaqwen_amd.decoder import MegakernelPrefillDecoder
+    dec, _, sp, _ = mid
     toks = make_tokens(n, sp["vocab_size"], seed=n)
     dec.reset()
     _, want = dec.prefill_step_with_logits(toks)
     tight = MegakernelPrefillDecoder(dec.embed_weight, dec.layer_weights, dec.final_norm_weight,
-                                     dec.lm_head_weight, dec.cos_table, dec.sin_table, 2, 640,
+                                     dec.lm_head_weight, dec.cos_table, dec.sin_table, 2, 840,
                                      max_prefill_len=n)
+    # the workspace's tail: fp32 buffers of 64 positions (residual stream before and after each
+    # sub-block, q|k|v, attention output, MLP vector) and 8 claim counters of 128 bytes
+    fused = 64 * 4 * ((2 * 2 + 1) * 1024 + 2 * (4096 + 2048 + 3072)) + 8 * 128
+    total = _lib.load().mq_workspace_bytes(ctypes.byref(tight._desc))
+    desc = _lib.ModelDesc.from_buffer_copy(tight._desc)
+    desc.max_prefill_len = 0
+    tiles = (n + 31) // 32
+    other = sum((n * w * 2 + 255) // 256 * 256 for w in (1024, 1024, 4096, 2048, 3072)) \
+        + 2 * 8 * tiles * 4096 * 2
+    sums = total - fused - _lib.load().mq_workspace_bytes(ctypes.byref(desc)) - other
+    assert sums > 0 and sums % 4096 == 0           # whole fp32 rows: the tail starts behind them
+    tail = tight._workspace.view(torch.uint8)[total - fused:total]
+    tail.fill_(0xA5)
     for _ in range(2):
         _, got = tight.prefill_step_with_logits(toks)
         assert torch.equal(got, want)
         assert torch.equal(tight.k_cache[:, :, :n], dec.k_cache[:, :, :n])
         assert torch.equal(tight.v_cache[:, :, :n], dec.v_cache[:, :, :n])
+        assert bool((tail == 0xA5).all())
     dec.reset()
-
-
-@pytest.fixture(scope="module")
-def mid():
-    return build_pair(2, 4096, 840, seed=5, norm_jitter=0.1, max_prefill=832)
 
 
 @pytest.mark.parametrize("n", [1, 63, 65, 256, 257, 512, 513, 768, 769, 832])
