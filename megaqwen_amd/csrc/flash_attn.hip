@@ -23,9 +23,12 @@
 // What bounds it: a (32 queries, 32 keys) unit is 12 MFMAs (384 matrix cycles) and ~105 VALU
 // instructions, 16 of them exponentials, which a SIMD issues in ~480 cycles; a loop of just that
 // mix, interleaved, runs 550-600 cycles per unit.  The matrix products of one unit are therefore
-// interleaved with the weights of another.  T = 1500, 14 heads, bf16: 27.4 -> 22 us per call; 4 x
-// 14 heads, T = 3000, fp16: 272 -> 228 us, at a clock the power limit holds near 1.7 GHz (2.05 for
-// the register-only loop).
+// interleaved with the weights of another.  Neither shape below reaches that loop:
+//   14 heads, T = 1500, bf16 (25.4 -> 20.8 us per call): one round of 658 workgroups, ~30 units per
+//     SIMD; 19% MFMA-busy, the waves wait on memory for 28% of their cycles (a tile is copied half a
+//     unit before the wait for it) and issue in 35%;
+//   4 x 14 heads, T = 3000, fp16 (271 -> 226 us): 43% MFMA-busy, ~910 cycles per unit at 1.9 GHz, a
+//     sixth of them because 2632 workgroups are 5.14 rounds run as 6.
 // Keys >= T (the last tile) get score -inf and zero V^T entries; queries >= T read row T-1 and
 // store nothing.  All accesses stay inside the tensors.
 #include <hip/hip_runtime.h>
@@ -37,7 +40,6 @@
 #include "mq_flash.h"
 
 #define FA_D 64           // head dim
-#define FA_QB 32          // queries per workgroup
 #define FA_KT 32          // keys per tile
 #define FA_WAVES 4        // waves per workgroup (split of the key tiles)
 // N groups of one MFMA followed by V VALU instructions
@@ -86,8 +88,9 @@ template <bool HI> MQ_DEV float fa_extreme(float a, float b) {
   else return __builtin_elementwise_minimum(a, b);
 }
 
-// Two weights as packed 16-bit hi parts (truncated, so that lo is never negative and an infinite
-// v gives an infinite, not a NaN, output) and lo parts (the exact remainder p - hi, rounded once).
+// Two weights as packed 16-bit hi parts (truncated, so that lo is never negative) and lo parts (the
+// exact remainder p - hi, rounded once).  An infinite v gives an infinite output where lo is not 0;
+// where the weight is exact in 16 bits (T = 1, say) lo is 0 and the output NaN.
 // The remainder is one instruction per weight: a two-element dot product of the packed
 // hi pair with (-1, 0) or (0, -1) plus p, or a mixed-precision fma for fp16.
 template <bool F16> MQ_DEV void fa_split2(float p0, float p1, uint32_t& hi, uint32_t& lo) {
@@ -538,12 +541,14 @@ int mq_launch_flash_attn_bhwd(const void* q, const void* k, const void* v, void*
   const uint16_t* kk = static_cast<const uint16_t*>(k);
   const uint16_t* vv = static_cast<const uint16_t*>(v);
   uint16_t* oo = static_cast<uint16_t*>(out);
-  // 64 queries per wave move half the operand bytes per query, which pays once the chip is power
-  // and issue bound, but come in units twice as large.  So by rounds of resident workgroups (768
-  // of 32 queries, 512 of 64): 64 queries when that takes fewer rounds, or as many with the
-  // last round of the 32-query grid nearly full.  Measured per call, 14 heads, 32 against 64
-  // queries: T 1500 22.8 / 25.6 us, T 1800 33.6 / 30.3, T 2600 56.0 / 60.0, T 3000 74.0 / 67.8,
-  // 4 x T 700 22.1 / 24.1, 4 x T 3000 251.6 / 235.6.
+  // 64 queries per wave move half the operand bytes per query, but come in units twice as large.
+  // So by rounds of resident workgroups on 256 CUs (3 of 32 queries per CU, 2 of 64): 64 queries when
+  // that takes fewer rounds, or as many, more than one, with the last round of the 32-query grid
+  // more than 65% full: above two thirds it puts a third workgroup on CUs.  Measured per call, 32
+  // against 64 queries (us), with the fill of the last 32-query round: 14 heads T 2592 (48%) 52.9 /
+  // 55.2, T 2848 (62%) 59.2 / 60.2, T 2912 (66%) 60.8 / 61.2, T 2976 (70%) 69.2 / 62.9; 28 heads T 1440
+  // (64%) 33.8 / 35.0, T 1480 (71%) 39.5 / 36.4; 56 heads T 704 (60%) 20.4 / 21.7, T 736 (68%) 23.5 /
+  // 22.0, T 1153 (70% of a third round) 47.1 / 46.2; fewer rounds: 42 heads T 1500 53.2 / 46.7.
   const long long i1 = (long long)bh * ((T + 31) / 32), i2 = (long long)bh * ((T + 63) / 64);
   const long long r1 = (i1 + 767) / 768, r2 = (i2 + 511) / 512;
   const bool wide = r2 < r1 || (r2 == r1 && r1 > 1 && 20 * i1 > 768 * (20 * r1 - 7));

@@ -211,7 +211,7 @@ static_assert(512 / GEMM_BK % GEMM_STAGES == 0 && 512 / GEMM_BK % GEMM_STAGES_BI
 //            used when there are enough of them to fill the CUs).
 //   BM = 32 (BN = 64): waves 0/1 and 2/3 compute the same two 32 x 32 blocks over the first and
 //            the second half of every K step; the halves are added in LDS before the epilogue
-//            (this doubles the workgroups of the N = 1024 GEMMs at M = 512).
+//            (twice the workgroups of 64 x 64 tiles, for the N = 1024 GEMMs of 769..960 rows).
 // Epilogue of a q or k head tile of the q|k|v GEMM (the work of prefill_qk_norm_rope_kernel,
 // fused_prefill_kernels.inl:112-258): the bf16-rounded tile goes through LDS (row stride 136
 // bf16), then 16 threads per position take dims 4i .. 4i + 3 and their RoPE partners
@@ -854,7 +854,9 @@ static GemmPlan gemm_plan(int M, int N) {
 // the residual epilogue need, whose loads bound them; the sums cost 4 KB per row and split once
 // out and in.  Per layer, O + down, residual epilogue -> split (us, one card): 32 rows -4.5, 128
 // -5.2, 256 -5.5, 384 -2.3, 512 -1.1, 640 -4.9, 768 -4.5; at 1024 rows, where 64 x 64 tiles alone
-// fill the CUs, +1.9.
+// fill the CUs, +1.9.  Between, 2 splits of 64 x 128 tiles would gain too (4-layer prefill, residual
+// epilogue -> split, us: 769 rows 436 -> 421, 832 439 -> 425, 960 448 -> 437, 961 437 -> 444, 1024 438 ->
+// 448), so the line could move to 960.
 struct PartPlan {
   int rows;          // the longest prompt the plan serves
   int bn, sk;        // tile columns and splits

@@ -82,10 +82,11 @@ def test_op_decode_layer_matches_oracle_and_decoder(pair):
     dec.check()
 
 
-# both sides of the one-block (224 positions) / split switch and of a chunk's edge; in the split
-# form the last chunk may hold the new position alone (225, 449), and at 7169 and above every
-# chunk spans more than one 224-position block
-@pytest.mark.parametrize("pos", [0, 1, 222, 223, 224, 225, 447, 448, 449, 1500, 7168, 7300])
+# both sides of the one-block (224 positions) / split switch and of steps of the chunk length; the
+# new position is in the last chunk.  At 7169 and 7301 positions (32 chunks) every chunk but the last,
+# of 194 and 202, spans two 224-position blocks; at 7424 the last one does too, with the new position
+# in its second block
+@pytest.mark.parametrize("pos", [0, 1, 222, 223, 224, 225, 447, 448, 449, 1500, 7168, 7300, 7423])
 def test_op_decode_layer_attention_split(pos):
     """mq_op_decode_layer over a random cache against the oracle layer, the written K/V rows
     included and no other row touched."""

@@ -90,8 +90,8 @@ def test_peaked_softmax(dtype):
 @pytest.mark.parametrize("bh,t", [(3, 31), (3, 32), (3, 33), (2, 64), (2, 65), (3, 127), (2, 129),
                                   (1, 161), (400, 33), (400, 64), (220, 97), (160, 129),
                                   (130, 191)])
-@pytest.mark.parametrize("dtype,scale", [(torch.bfloat16, 0.125), (torch.float16, -0.2),
-                                         (torch.bfloat16, 0.0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("scale", [0.125, -0.2, 0.0])
 def test_tile_edges(bh, t, dtype, scale):
     q, k, v = _inputs((1, bh, t, 64), dtype, seed=bh + t)
     out = _fa()(q.cuda(), k.cuda(), v.cuda(), scale=scale)
@@ -99,12 +99,42 @@ def test_tile_edges(bh, t, dtype, scale):
     _check(out.cpu(), q, k, v, scale)
 
 
-def test_unaligned_and_non_finite_inputs():
+# 64 queries per workgroup, 6 to 15 key tiles per wave: tiles copied two ahead are used, and T % 32
+# != 0 leaves a partial last tile.  mag 6 with keys that grow along T: scores of later tiles exceed
+# the softmax reference again and again, so that sums other than zero are rescaled
+@pytest.mark.parametrize("bh,t", [(56, 781), (56, 1001), (14, 1801)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("scale,mag", [(0.125, 1.0), (-0.2, 1.0), (0.125, 6.0), (-0.125, 6.0)])
+def test_wide_workgroups(bh, t, dtype, scale, mag):
+    q, k, v = _inputs((1, bh, t, 64), torch.float32, seed=bh + t)
+    if mag != 1.0:
+        k = k * torch.linspace(0.2, 1.0, t)[:, None] * mag
+        q = q * mag
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    out = _fa()(q.cuda(), k.cuda(), v.cuda(), scale=scale)
+    torch.cuda.synchronize()
+    _check(out.cpu(), q, k, v, scale)
+
+
+def test_one_key():
+    """T = 1: the weight is exactly 1, so the output is v (an infinite v gives no finite output:
+    its dim meets the weight's lo part, 0)."""
+    q, k, v = _inputs((1, 3, 1, 64), torch.bfloat16, seed=4)
+    assert torch.equal(_fa()(q.cuda(), k.cuda(), v.cuda()).cpu(), v)
+    v[0, 1, 0, 9] = float("inf")
+    got = _fa()(q.cuda(), k.cuda(), v.cuda()).cpu()
+    assert not torch.isfinite(got[0, 1, 0, 9])
+    got[0, 1, 0, 9] = v[0, 1, 0, 9]
+    assert torch.equal(got, v)
+
+
+# 32 queries per workgroup, and 64
+@pytest.mark.parametrize("bh,t", [(2, 70), (56, 1001)])
+def test_unaligned_and_non_finite_inputs(bh, t):
     """Contiguous tensors that start 2 bytes into an allocation; an infinite value reaches only
     its own dim's outputs, a NaN query only its own row, and the rows past T of the last key tile
     (T % 32 != 0) add nothing."""
-    t = 70
-    q, k, v = _inputs((1, 2, t, 64), torch.bfloat16, seed=21)
+    q, k, v = _inputs((1, bh, t, 64), torch.bfloat16, seed=21)
     dev = []
     for x in (q, k, v):
         buf = torch.zeros(x.numel() + 1, dtype=x.dtype, device="cuda")
