@@ -1862,8 +1862,8 @@ __global__ void __launch_bounds__(MQ_THREADS) mq_op_merge_kernel(MqDecodeParams 
 }
 // The middle of one whole layer (mq_launch_op_layer): q/k RMSNorm, RoPE, the K/V cache row,
 // attention over [0, pos] and the O projection, split by kv head as in the persistent kernel
-// (workgroup wg serves head wg % 8; the 8 partial O vectors go to s->opart and the MLP kernels add
-// them to the layer input).  Every attention workgroup normalises and rotates its head's q and k
+// (workgroup wg serves head wg % 8; the 8 partial O vectors go to s->opart and the gate|up kernel
+// adds them to the layer input).  Every attention workgroup normalises and rotates its head's q and k
 // itself, so no kernel stands between the projection and the attention.
 // Up to one 224-position block, every workgroup of a head attends over all positions and goes
 // straight on to its O rows (LOCAL); above it, chunks of the positions are attended by
