@@ -28,7 +28,7 @@
 //     SIMD; 19% MFMA-busy, the waves wait on memory for 28% of their cycles (a tile is copied half a
 //     unit before the wait for it) and issue in 35%;
 //   4 x 14 heads, T = 3000, fp16 (271 -> 226 us): 43% MFMA-busy, ~910 cycles per unit at 1.9 GHz, a
-//     sixth of them because 2632 workgroups are 5.14 rounds run as 6.
+//     seventh of them because 2632 workgroups are 5.14 rounds run as 6.
 // Keys >= T (the last tile) get score -inf and zero V^T entries; queries >= T read row T-1 and
 // store nothing.  All accesses stay inside the tensors.
 #include <hip/hip_runtime.h>
