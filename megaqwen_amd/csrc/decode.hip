@@ -1944,11 +1944,14 @@ __global__ void __launch_bounds__(MQ_THREADS) mq_op_layer_gateup_kernel(MqDecode
   gu_load(ws, p.layers[l], blockIdx.x, gridDim.x);
   reinterpret_cast<float2*>(lds + LDS_IN)[tid()] = op_layer_a2(p, x, 2 * tid());
   __syncthreads();
-  int r0, nr;
-  hid_rows(blockIdx.x, gridDim.x, r0, nr);
-  if (tid() < nr) st_coh(p.s->a + r0 + tid(), lds[LDS_IN + r0 + tid()]);
   gu_run(ws, p.layers[l], blockIdx.x, gridDim.x, lds);
-  phase_finish([&] { gu_publish_f(p.s->mlp, blockIdx.x, gridDim.x, lds); });
+  phase_finish([&] {
+    int r0, nr;
+    hid_rows(blockIdx.x, gridDim.x, r0, nr);
+    const int t = lane_id();
+    if (t < nr) st_coh(p.s->a + r0 + t, lds[LDS_IN + r0 + t]);
+    gu_publish_f(p.s->mlp, blockIdx.x, gridDim.x, lds);
+  });
 }
 // (c) SwiGLU MLP with residual: x_out = bf16(W_d (silu(W_g n) * W_u n) + a), n = RMSNorm(a).
 __global__ void __launch_bounds__(MQ_THREADS) mq_op_gateup_kernel(MqDecodeParams p, int l,
